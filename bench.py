@@ -484,7 +484,7 @@ def main():
                 ("gemm_q8_0_k4096_rows4096_N512", G.GgmlType.Q8_0, 4096, 4096, 512, S.q8_0_matrix, True),
                 ("gemm_iq2_xxs_k4096_rows1536_N64", G.GgmlType.IQ2_XXS, 1536, 4096, 64, iq, True)]:
             r = run_gemm(L, s, ty, rows, K, N, mk, max(20, args.steps // 5), max(5, args.warmup // 5), 9, use_work=uw)
-            r["path"] = ["f16 MFMA tiles", "f16 MFMA tiles (K split)", "f16 dequant + hipBLASLt"][
+            r["path"] = ["f16 MFMA tiles", "f16 MFMA tiles (K split)", "many-token workspace path"][
                 G.ops.gemm_path(ty, K, rows, N, G.row_bytes(ty, K), rows, r["workspace_bytes"])]
             secondary[name] = r
             log(f"{name}: {r}")

@@ -12,6 +12,12 @@ gs_blob_##NAME##_end:                    \
 BLOB(common, "build/common.hsaco")
 BLOB(grouped, "build/grouped.hsaco")
 BLOB(gemm, "build/gemm.hsaco")
+BLOB(q8, "build/q8.hsaco")
+BLOB(q12, "build/q12.hsaco")
+BLOB(q13, "build/q13.hsaco")
+BLOB(q14, "build/q14.hsaco")
+BLOB(q16, "build/q16.hsaco")
+BLOB(q18, "build/q18.hsaco")
 BLOB(t0, "build/t0.hsaco")
 BLOB(t1, "build/t1.hsaco")
 BLOB(t8, "build/t8.hsaco")

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -29,7 +30,7 @@
 #define GS_BLOB(NAME)                                 \
     extern "C" const unsigned char gs_blob_##NAME##_start[]; \
     extern "C" const unsigned char gs_blob_##NAME##_end[];
-#define GS_BLOB_LIST(X) X(common) X(grouped) X(gemm) X(t0) X(t1) X(t8) X(t10) X(t11) X(t12) X(t13) X(t14) X(t16) X(t18) X(t22) X(t23) X(t30)
+#define GS_BLOB_LIST(X) X(common) X(grouped) X(gemm) X(q8) X(q12) X(q13) X(q14) X(q16) X(q18) X(t0) X(t1) X(t8) X(t10) X(t11) X(t12) X(t13) X(t14) X(t16) X(t18) X(t22) X(t23) X(t30)
 GS_BLOB_LIST(GS_BLOB)
 
 namespace {
@@ -852,6 +853,124 @@ int gemm_lib(DeviceCtx *c, int ty, const uint8_t *W, int K, int rows, const floa
     return hipSuccess;
 }
 
+// ---- quantized GEMM kernels (qgemm.hip) -----------------------------------------------------------
+struct QgShape {
+    int nr, nt, rg, kg, xh;   // kernel: 16 nr rg rows x 16 nt tokens; xh: activations as f16 slabs from the workspace
+    int slices;               // K slices (blockIdx.z), partial tiles in the workspace
+    double us;                // modelled time
+};
+struct QgFmt {
+    int slot, table;          // bytes of a super-block's LDS slot and of the decode tables
+    bool dwords;              // rows start on dwords (formats whose super-block is whole dwords)
+    double cost;              // decode cost against Q4_K, from measured calls
+};
+const QgFmt *qg_fmt(int ty) {
+    static const std::map<int, QgFmt> f = {{GS_Q8_0, {272, 0, true, 1.15}},     {GS_Q4_K, {144, 0, true, 1.0}},
+                                           {GS_Q5_K, {176, 0, true, 1.1}},      {GS_Q6_K, {240, 0, false, 1.25}},
+                                           {GS_IQ2_XXS, {80, 5120, false, 1.15}}, {GS_IQ3_XXS, {112, 3072, false, 1.3}}};
+    const auto it = f.find(ty);
+    return it == f.end() ? nullptr : &it->second;
+}
+// LDS of a kernel: tables, the activation buffers, two buffers of the raw chunk; at least the partial
+// tiles of the end (qgemm.hip has the same figures)
+size_t qg_lds(const QgFmt &f, const QgShape &q) {
+    const int hs = q.kg == 8 ? 2 : 1, rc = q.kg != 8 ? 1 : q.nr == 1 ? 4 : f.slot >= 176 ? 2 : 4;
+    const size_t raw = ((size_t)16 * q.nr * q.rg * rc * f.slot + 1023) / 1024 * 1024;
+    const size_t xb = (size_t)q.nt * 4096 * hs, base = f.table + 2 * raw;
+    const size_t run = base + (q.xh && base + 3 * xb + 64 <= 160 * 1024 ? 3 : 2) * xb;
+    const size_t wb = (size_t)q.nr * q.nt * 1024, end = (q.kg == 2 ? q.rg : 8) * wb;
+    return std::max(run, end);
+}
+size_t qg_x16_bytes(const QgShape &q, int K, int N, int n_batch) {
+    const int T = 16 * q.nt;
+    return q.xh ? a256((size_t)n_batch * ((N + T - 1) / T) * T * K * 2) : 0;
+}
+// The kernel for a problem, or slices = 0 where another path is faster. Each path's time is modelled
+// from measured calls (us, one MI355X, Q4_K; 12288 x 4096, 4096 x 4096, 4096 x 12288 and 2048 x 2048
+// at 9 .. 512 tokens, all six formats): a start-up, then rounds over the CUs x super-blocks per slice
+// x a cost per super-block, and the slices' sum. The lines between the paths follow from it:
+//   tiles of 16 .. 48 rows x all tokens (kg 8), up to 96 tokens a block. 12288 x 4096: 16 tokens 28 ->
+//     18 us, 77 tokens 44 -> 24 (28 without a workspace for f16 activations); 4096 x 12288 x 77, two K
+//     slices, 39 -> 31; fewer tokens of long narrow matrices stay on the 128 x 64 tiles' K split
+//     (4096 x 12288 x 48: 27);
+//   tiles of 128 or 192 rows x 128 tokens (kg 2) with the many-token workspace: 12288 x 4096 x 256
+//     65 -> 48 us, x 512 76 -> 64; 4096 x 12288 x 256, four slices, 70 -> 48, x 512, two, 97 -> 82.
+//     Dequantization + library GEMM stays where tiles are few for the tokens: 4096 x 4096 x 512 (41
+//     against 43), 2048 x 2048 from 256 tokens (20 against 24).
+QgShape qg_pick(DeviceCtx *c, int ty, const void *W, int64_t row_stride, int64_t w_bs, int K, int rows, int N, int n_batch,
+                int64_t x_stride, size_t work_bytes, bool lib) {
+    QgShape best{0, 0, 0, 0, 0, 0, 0.0};
+    const QgFmt *f = qg_fmt(ty);
+    if (!f || K % 256 != 0 || row_stride < 0 || (f->dwords && (((uintptr_t)W | (uintptr_t)row_stride | (uintptr_t)w_bs) & 3))) return best;
+    const int nsb = K / 256, cus = c->cu_count;
+    auto rounds = [&](int64_t wgs) { return (double)((wgs + cus - 1) / cus); };
+    // 32-bit offsets within a tile's rows and a token block's activations
+    if (((int64_t)192 * row_stride + (int64_t)nsb * 272) >> 32 || x_stride < 0 || ((int64_t)128 * x_stride + K) * 4 >> 32) return best;
+    // the paths without these kernels
+    const double W1 = (double)rows * K * n_batch;
+    int ksb = 0;
+    const int nks = work_bytes > 0 ? gemm_slices(c, K, rows, N, n_batch, &ksb) : (ksb = nsb, 1);
+    const int64_t tiles = (int64_t)((rows + 127) / 128) * ((N + 63) / 64) * n_batch * nks;
+    double limit = lib ? 15.5 + 0.5e-6 * W1 + 3.0 * std::pow(2e-9 * N * W1, 0.63)
+                       : 6 + (nks > 1 ? 5 : 0) + rounds(tiles) * ksb * f->cost * (N > 64 ? 2.4 : 1.4 + 0.006 * N);
+    limit *= 0.97;
+    auto consider = [&](QgShape q, double t0, double per) {
+        const int64_t T = 16 * q.nt, RB = 16 * (int64_t)q.nr * q.rg, wg1 = (rows + RB - 1) / RB * ((N + T - 1) / T) * n_batch;
+        for (int s = 1; s <= GS_GEMM_KS_MAX && s <= nsb; s++) {
+            q.slices = s;
+            const int ks = (nsb + s - 1) / s;
+            if ((nsb + ks - 1) / ks != s) continue;   // fewer slices do the same
+            const size_t part = s > 1 ? gemm_part_bytes(s, rows, N, n_batch) : 0;
+            if (qg_x16_bytes(q, K, N, n_batch) + part > work_bytes) {
+                if (q.xh || s > 1) break;
+            }
+            q.us = t0 + rounds(wg1 * s) * ks * per * f->cost + (s > 1 ? 3 + (double)s * N * rows * n_batch * 2e-6 : 0);
+            if (q.us < limit && (best.slices == 0 || q.us < best.us)) best = q;
+            if (wg1 * s >= 2 * cus) break;
+        }
+    };
+    if (N <= 192) {
+        const int nb = (N + 95) / 96, nt = ((N + nb - 1) / nb + 15) / 16;   // token blocks of even size
+        consider({1, nt, 1, 8, 0, 0, 0}, 3.0, 0.456 + 0.115 * nt);
+        consider({2, nt, 1, 8, 0, 0, 0}, 3.5, 0.55 + 0.155 * nt);
+        consider({3, nt, 1, 8, 0, 0, 0}, 4.0, 0.66 + 0.18 * nt);
+        consider({2, nt, 1, 8, 1, 0, 0}, 6.5, 0.49 + 0.065 * nt);
+        consider({3, nt, 1, 8, 1, 0, 0}, 6.5, 0.64 + 0.095 * nt);
+    }
+    if (N > 64) {
+        consider({2, 8, 4, 2, 0, 0, 0}, 9.0, 2.6);
+        consider({2, 8, 4, 2, 1, 0, 0}, 11.0, 2.4);
+        if (ty != GS_Q8_0) consider({3, 8, 4, 2, 1, 0, 0}, 11.0, 3.3);   // (Q8_0: its raw chunks do not fit)
+    }
+    return best;
+}
+int qg_launch(DeviceCtx *c, int ty, const QgShape &q, QGemmArgs g, int n_batch, void *work, hipStream_t s) {
+    const int T = 16 * q.nt, RB = 16 * q.nr * q.rg, nsb = g.K / 256;
+    g.n_rb = (g.rows + RB - 1) / RB;
+    g.n_tb = (g.N + T - 1) / T;
+    g.ksb = (nsb + q.slices - 1) / q.slices;
+    // row block r runs on XCD r % 8 (workgroup w -> XCD w % 8), its token blocks back to back
+    const int64_t nwg = (int64_t)8 * ((g.n_rb + 7) / 8) * g.n_tb;
+    if (nwg > 0x7fffffff) return hipErrorInvalidValue;
+    hipError_t e;
+    if (q.xh) {
+        g.X16 = (const uint16_t *)work;
+        QGemmXArgs x{g.X, (uint16_t *)work, g.x_stride, g.x_bs, g.K, g.N, T, g.n_tb};
+        const int64_t thr = (int64_t)g.N * (g.K / 8);
+        if ((e = launch("gs_k_qgemm_x", dim3((unsigned)((thr + 255) / 256), n_batch), dim3(256), 0, s, x)) != hipSuccess) return e;
+    }
+    if (q.slices > 1) g.part = (float *)((uint8_t *)work + qg_x16_bytes(q, g.K, g.N, n_batch));
+    const std::string name = "gs_k_qgemm_" + std::to_string(ty) + "_" + std::to_string(q.nr) + "_" + std::to_string(q.nt) + "_" +
+                             std::to_string(q.rg) + "_" + std::to_string(q.kg) + "_" + std::to_string(q.xh);
+    e = launch(name, dim3((unsigned)nwg, n_batch, q.slices), dim3(512), qg_lds(*qg_fmt(ty), q), s, g);
+    if (e == hipSuccess && q.slices > 1) {
+        GemmReduceArgs r{g.part, g.Y, g.y_stride, g.y_bs, g.rows, g.N, n_batch, q.slices, g.accumulate};
+        const int64_t total = (int64_t)n_batch * g.N * g.rows;
+        e = launch("gs_k_gemm_reduce", dim3((unsigned)std::min<int64_t>((total + 255) / 256, 4 * (int64_t)c->cu_count)), dim3(256), 0, s, r);
+    }
+    return e;
+}
+
 int gemm_impl(int ty, const void *W, int64_t row_stride, int K, int rows, const float *X, int64_t x_stride, float *Y,
               int64_t y_stride, int N, int accumulate, int n_batch, int64_t w_bs, int64_t x_bs, int64_t y_bs,
               void *work, size_t work_bytes, void *s) {
@@ -895,10 +1014,22 @@ int gemm_impl(int ty, const void *W, int64_t row_stride, int K, int rows, const 
     hipError_t e;
     DeviceCtx *c = ctx(&e);
     if (!c) return e;
+    const bool lib = work && aligned16(work) && gemm_lib_eligible(ty, K, rows, N, row_stride, y_stride, work_bytes);
+    int ksb = 0;
+    const int nks = work ? gemm_slices(c, K, rows, N, n_batch, &ksb) : 1;
+    // a workspace that is too small for the K split is refused
+    if (!lib && nks > 1 && (work_bytes < gemm_part_bytes(nks, rows, N, n_batch) || !aligned16(work))) return hipErrorInvalidValue;
+    const QgShape q = qg_pick(c, ty, W, row_stride, n_batch > 1 ? w_bs : 0, K, rows, N, n_batch, x_stride,
+                              work && aligned16(work) ? work_bytes : 0, lib);
+    if (q.slices) {
+        QGemmArgs g{(const uint8_t *)W, X, nullptr, Y, nullptr, row_stride, x_stride, y_stride, w_bs, x_bs, y_bs,
+                    K, rows, N, accumulate, 0, 0, 0, a.wait_limit, a.wait_force};
+        return qg_launch(c, ty, q, g, n_batch, work, (hipStream_t)s);
+    }
     // many tokens and a workspace for the f16 operands: dequantize + library GEMM (contiguous rows;
     // every block format, and F16 weights as they are: Q8_0 too, whose tile decode is the cheapest,
     // 42 against 50 us at 4096 x 4096 x 512 and 82 against 137 us at 12288 x 4096 x 512)
-    if (work && aligned16(work) && gemm_lib_eligible(ty, K, rows, N, row_stride, y_stride, work_bytes)) {
+    if (lib) {
         const int r = gemm_lib(c, ty, (const uint8_t *)W, K, rows, X, x_stride, Y, y_stride, N, accumulate, n_batch, w_bs,
                                x_bs, y_bs, work, (hipStream_t)s);
         if (r >= 0) return r;
@@ -907,11 +1038,8 @@ int gemm_impl(int ty, const void *W, int64_t row_stride, int K, int rows, const 
     // K split only into the caller's workspace: each slice writes its f32 partial tile there and
     // gs_k_gemm_reduce sums the slices in slice order into Y (a fixed order, so the result is
     // reproducible). Without a workspace the whole K runs in one tile pass.
-    int ksb = 0;
-    const int nks = work ? gemm_slices(c, K, rows, N, n_batch, &ksb) : 1;
     if (nks == 1)
         return launch(name, dim3((unsigned)nwg, n_batch, 1), dim3(GS_GEMM_THREADS, 1, 1), lds, (hipStream_t)s, a);
-    if (work_bytes < gemm_part_bytes(nks, rows, N, n_batch) || !aligned16(work)) return hipErrorInvalidValue;
     a.ksb = ksb;
     a.part = (float *)work;
     e = launch(name, dim3((unsigned)nwg, n_batch, nks), dim3(GS_GEMM_THREADS, 1, 1), lds, (hipStream_t)s, a);
@@ -947,7 +1075,8 @@ GS_EXPORT int gs_gemm_path(int ty, int K, int rows, int N, int64_t row_stride, i
     hipError_t e;
     DeviceCtx *c = ctx(&e);
     if (!c) return -(int)e;
-    if (gemm_lib_eligible(ty, K, rows, N, row_stride, y_stride, work_bytes) && lt_plan(c, K, rows, N, y_stride))
+    if (gemm_lib_eligible(ty, K, rows, N, row_stride, y_stride, work_bytes) &&
+        (qg_pick(c, ty, nullptr, row_stride, 0, K, rows, N, 1, K, work_bytes, true).slices || lt_plan(c, K, rows, N, y_stride)))
         return 2;
     int ksb = 0;
     return work_bytes > 0 && gemm_slices(c, K, rows, N, 1, &ksb) > 1 &&

@@ -170,3 +170,24 @@ struct GemmReduceArgs {
     int64_t y_stride, y_bs;
     int rows, N, n_batch, nks, accumulate;
 };
+
+// Quantized GEMM in row tiles (qgemm.hip): the product of GemmArgs
+struct QGemmArgs {
+    const uint8_t *W;
+    const float *X;           // f32 rows (kernels with XH = 0)
+    const uint16_t *X16;      // f16 half slabs [batch][token block][K / 128][16 NT tokens][16 chunks, swizzled]
+    float *Y;
+    float *part;              // K split: slice partials [slice][batch][N][rows] (null: write Y)
+    int64_t row_stride, x_stride, y_stride;
+    int64_t w_bs, x_bs, y_bs;
+    int K, rows, N, accumulate;
+    int n_rb, n_tb, ksb;      // row blocks, token blocks, super-blocks per K slice
+    uint32_t wait_limit, wait_force;
+};
+// f32 rows -> QGemmArgs::X16
+struct QGemmXArgs {
+    const float *x;
+    uint16_t *y;
+    int64_t x_stride, x_bs;
+    int K, N, T, n_tb;
+};

@@ -1215,6 +1215,21 @@ extern "C" __global__ void __launch_bounds__(256) gs_k_f32_to_f16(EltArgs a) {
 extern "C" __global__ void __launch_bounds__(256) gs_k_rows_to_f16(CvtArgs a) {
     rows_to_f16(a.x, a.y, a.x_stride, a.K, a.N, (int64_t)blockIdx.x * blockDim.x + threadIdx.x);
 }
+// activations of the quantized GEMM (qgemm.hip): 8 values per thread, f32 -> f16 (round to nearest
+// even), token blocks of T rows as half slabs [K / 128][T][256 bytes], chunk c of token t at c ^ (t & 15)
+extern "C" __global__ void __launch_bounds__(256) gs_k_qgemm_x(QGemmXArgs a) {
+    typedef float f8v __attribute__((ext_vector_type(8)));
+    typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int per = a.K / 8, z = blockIdx.y;
+    if (i >= (int64_t)per * a.N) return;
+    const int n = (int)(i / per), kc = (int)(i - (int64_t)n * per), tb = n / a.T, t = n - tb * a.T;
+    const float4 *src = (const float4 *)(a.x + (int64_t)z * a.x_bs + (int64_t)n * a.x_stride + 8 * kc);
+    const float4 p0 = src[0], p1 = src[1];
+    const f8v v = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+    uint8_t *dst = (uint8_t *)a.y + (((int64_t)(z * a.n_tb + tb) * (a.K / 128) + (kc >> 4)) * a.T + t) * 256;
+    *(h8v *)(dst + (((kc & 15) ^ (t & 15)) << 4)) = __builtin_convertvector(v, h8v);
+}
 extern "C" __global__ void __launch_bounds__(256) gs_k_saxpy(EltArgs a) {  // y = s*x + y
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < a.n) a.y[i] = a.s * a.a[i] + a.y[i];

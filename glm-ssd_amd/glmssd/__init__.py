@@ -314,7 +314,7 @@ class ops:
 
     @staticmethod
     def gemm_path(ty, k, rows, n, row_stride, y_stride, work_bytes):
-        """gs_gemm_path: 0 f16 MFMA tiles, 1 tiles with the K split, 2 f16 dequant + hipBLASLt."""
+        """gs_gemm_path: 0 MFMA tiles, 1 with the K split into the workspace, 2 the many-token workspace path."""
         r = lib().gs_gemm_path(int(ty), k, rows, n, row_stride, y_stride, work_bytes)
         if r < 0:
             check(-r)

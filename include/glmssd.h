@@ -138,26 +138,27 @@ int gs_axpy(float *y, const float *x, float a, int64_t n, void *s);
  * Like the reference, allocates nothing and never synchronizes. */
 int gs_gemm(int ty, const void *W, int64_t row_stride, int K, int rows, const float *X, int64_t x_stride, float *Y,
             int64_t y_stride, int N, int accumulate, int n_batch, int64_t w_bs, int64_t x_bs, int64_t y_bs, void *s);
-/* Additive (no counterpart in the reference): gs_gemm with a caller-owned workspace, used two ways.
- * (1) Problems with few 128-row x 64-token tiles (small N, few rows) split K across workgroups:
- * each slice writes its f32 partial tile into `work` and the slices are added in a fixed order.
- * (2) From N = 256 tokens (N > 128 for matrices of rows*K >= 2^25 weights), for every weight
- * type but F32 and BF16 and rows stored back to back (row_stride = bytes of a row), the weights are dequantized into `work` as f16 (F16 weights
- * are used in place), X is converted to f16 there too, and the product runs as an f16 x f16 -> f32
- * GEMM in hipBLASLt (the heuristic's first algorithm for the shape, so a shape always takes the
- * same one). Both round the operands to f16 exactly as gs_gemm does and accumulate in f32; results
- * repeat call to call and differ from gs_gemm only in f32 summation order. gs_gemm_workspace gives
- * the bytes a problem needs on the current device (0: `work` unused; for (2) rows*K*2 + N*K*2
- * rounded up to 256 each, plus 32 MiB of library workspace).
+/* Additive (no counterpart in the reference): gs_gemm with a caller-owned workspace, used for
+ * (1) the f32 partial tiles of a K split across workgroups, added in a fixed order (problems with few
+ * tiles: small N, few rows), (2) the f16 activations of the row-tile kernels, wherever the workspace
+ * holds them, and (3) from N = 256 tokens (N > 128 for matrices of rows*K >= 2^25 weights), every
+ * weight type but F32 and BF16 and rows stored back to back (row_stride = bytes of a row), either of
+ * those or the weights dequantized into `work` as f16 (F16 weights are used in place), X converted to
+ * f16 there too, and the product as an f16 x f16 -> f32 GEMM in hipBLASLt (the heuristic's first
+ * algorithm for the shape, so a shape always takes the same one); a rule on type, sizes and
+ * workspace_bytes picks the faster. Every path rounds the operands to f16 exactly as gs_gemm does and
+ * accumulates in f32; results repeat call to call and differ between paths only in f32 summation
+ * order. gs_gemm_workspace gives the bytes a problem needs on the current device (0: it needs none; a
+ * larger workspace may still be used; for (3) rows*K*2 + N*K*2 rounded up to 256 each, plus 32 MiB).
  * work: 16-byte aligned, >= that many bytes, not used by another call in flight; work == NULL
  * (or a smaller workspace) runs as gs_gemm. Never synchronizes; allocates nothing itself (the first
- * call of kind (2) on a device creates that device's hipBLASLt handle, kept until the process
+ * call that takes the library creates that device's hipBLASLt handle, kept until the process
  * ends). */
 int gs_gemm_workspace(int K, int rows, int N, int n_batch, size_t *bytes);
 /* Additive (no counterpart in the reference): the path gs_gemm_ex takes for a problem (one batch)
- * on the current device with a workspace of work_bytes: 0 the f16 MFMA tiles, 1 the tiles with the
- * K split, 2 the f16 dequant + hipBLASLt path (the library opens and has an algorithm for the
- * shape); a negative HIP error code if the device cannot run the library at all. */
+ * on the current device with a workspace of work_bytes: 0 MFMA tiles without the workspace's K split, 1
+ * with it, 2 the many-token path (f16 operands in the workspace, kind (3) above: the row-tile kernels, or
+ * the library where it opens and has an algorithm for the shape); a negative HIP error code if the device cannot run the library at all. */
 int gs_gemm_path(int ty, int K, int rows, int N, int64_t row_stride, int64_t y_stride, size_t work_bytes);
 int gs_gemm_ex(int ty, const void *W, int64_t row_stride, int K, int rows, const float *X, int64_t x_stride, float *Y,
                int64_t y_stride, int N, int accumulate, int n_batch, int64_t w_bs, int64_t x_bs, int64_t y_bs,
