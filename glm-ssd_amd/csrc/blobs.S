@@ -12,6 +12,7 @@ gs_blob_##NAME##_end:                    \
 BLOB(common, "build/common.hsaco")
 BLOB(grouped, "build/grouped.hsaco")
 BLOB(gemm, "build/gemm.hsaco")
+BLOB(mvgemv, "build/mvgemv.hsaco")
 BLOB(q8, "build/q8.hsaco")
 BLOB(q12, "build/q12.hsaco")
 BLOB(q13, "build/q13.hsaco")

@@ -30,7 +30,7 @@
 #define GS_BLOB(NAME)                                 \
     extern "C" const unsigned char gs_blob_##NAME##_start[]; \
     extern "C" const unsigned char gs_blob_##NAME##_end[];
-#define GS_BLOB_LIST(X) X(common) X(grouped) X(gemm) X(q8) X(q12) X(q13) X(q14) X(q16) X(q18) X(t0) X(t1) X(t8) X(t10) X(t11) X(t12) X(t13) X(t14) X(t16) X(t18) X(t22) X(t23) X(t30)
+#define GS_BLOB_LIST(X) X(common) X(mvgemv) X(grouped) X(gemm) X(q8) X(q12) X(q13) X(q14) X(q16) X(q18) X(t0) X(t1) X(t8) X(t10) X(t11) X(t12) X(t13) X(t14) X(t16) X(t18) X(t22) X(t23) X(t30)
 GS_BLOB_LIST(GS_BLOB)
 
 namespace {
@@ -291,6 +291,20 @@ bool stream_fits(int kind, int ty, StreamArgs a) {
     return plan_stream(c, kind, ty, a, P) == hipSuccess;
 }
 
+// formats of the row-tile GEMM (qgemm.hip) and, those without decode tables, of the several-vector
+// GEMV (mvgemv.hip)
+struct QgFmt {
+    int slot, table;          // bytes of a super-block's LDS slot and of the decode tables
+    bool dwords;              // rows start on dwords (formats whose super-block is whole dwords)
+    double cost;              // decode cost against Q4_K, from measured calls
+};
+const QgFmt *qg_fmt(int ty) {
+    static const std::map<int, QgFmt> f = {{GS_Q8_0, {272, 0, true, 1.15}},     {GS_Q4_K, {144, 0, true, 1.0}},
+                                           {GS_Q5_K, {176, 0, true, 1.1}},      {GS_Q6_K, {240, 0, false, 1.25}},
+                                           {GS_IQ2_XXS, {80, 5120, false, 1.15}}, {GS_IQ3_XXS, {112, 3072, false, 1.3}}};
+    const auto it = f.find(ty);
+    return it == f.end() ? nullptr : &it->second;
+}
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 int check_w(const void *W, int64_t row_stride) { return ((uintptr_t)W & 1) == 0 && (row_stride & 1) == 0; }
@@ -400,6 +414,65 @@ GS_EXPORT int gs_quant_q8_1(const float *x, void *q, int64_t n, void *s) {
 // =============================================================================================
 // GEMV (quants.cu:223-256)
 // =============================================================================================
+namespace {
+// Several vectors in one pass on int8 MFMA (mvgemv.hip), from this many. Measured against the streaming
+// kernels (which overlap their dot products with the weight stream, but hold few vectors' units in
+// registers: 5..8 vectors read the matrix twice, rows beyond 4096 elements once per vector).
+int mv_min(int ty, int K, int rows) {
+    const int64_t n = (int64_t)rows * K;
+    // rows beyond 4096: from 3, two vectors from about 2^24 weights (Q6_K 4096 x 6144: 9.0 us against
+    // 10.7, 512 x 12288 11.9 against 10.3; Q8_0 4096 x 6144 9.8 against 9.6, 4096 x 12288 16.2 against 21.2)
+    if (K > 4096) return n >= ((int64_t)1 << (ty == GS_Q8_0 ? 25 : 24)) ? 2 : 3;
+    if (ty == GS_Q8_0) return 3;
+    // Q6_K 2048 x 4096, 3 vectors: 7.7 against 7.7, 4 7.9 against 8.6; 1024 x 2048 6.0 against 5.6
+    if (ty == GS_Q6_K) return n >= ((int64_t)1 << 23) ? 3 : 5;
+    // Q4_K 12288 x 4096, 2 vectors: 11.9 against 10.6, 3 12.1 against 13.4; 4096 x 4096, 3 7.6 against
+    // 7.1, 4 7.7 against 7.7; 2048 x 4096, 4 7.5 against 6.9, 5 7.8 against 8.6
+    return n >= ((int64_t)1 << 25) ? 3 : n >= ((int64_t)1 << 24) ? 4 : 5;
+}
+struct MvPlan {
+    int depth = 0, grid = 0;
+    size_t lds = 0;
+};
+MvPlan mv_plan(DeviceCtx *c, int ty, MvArgs &m) {
+    MvPlan p;
+    const QgFmt *f = qg_fmt(ty);
+    if (!f || f->table || m.K % 256 != 0 || m.row_stride < 0 || (m.row_stride >> 26) || !aligned16(m.x) || m.x_stride % 4 != 0) return p;
+    if (f->dwords && (((uintptr_t)m.w | (uintptr_t)m.row_stride) & 3)) return p;
+    const int vg = m.nv <= 4 ? 1 : 2, nsb = m.K / 256;
+    const bool mins = ty == GS_Q4_K || ty == GS_Q5_K;
+    const size_t item = ((size_t)16 * f->slot + 1023) / 1024 * 1024, part = 2 * 8 * 256 * vg;
+    // the fewest chunks of K whose quantized vectors fit beside the rings; four items ahead where the
+    // smaller items leave room
+    for (int nc = 1; nc <= nsb && !p.depth; nc++) {
+        if (nsb % nc) continue;
+        const size_t U = m.K / nc / 32, xb = 64 + 32 * U * m.nv + (mins ? 2 : 1) * 16 * vg * U;
+        for (int d : {4, 2}) {
+            if (d == 4 && !mins) continue;
+            const size_t need = xb + part + 8 * d * item;
+            if (need > std::min<size_t>(c->max_lds, 160 * 1024) || p.depth) continue;
+            p.depth = d;
+            p.lds = need;
+            m.nchunk = nc;
+            m.ck = m.K / nc;
+        }
+    }
+    if (!p.depth) return p;
+    // waves along K against row tiles side by side: the fewest items for the busiest wave
+    const int ntile = (m.rows + 15) / 16, ns = m.ck / 256;
+    int64_t best = INT64_MAX;
+    for (int kg : {8, 4, 2, 1}) {
+        const int rg = 8 / kg, grid = std::min((ntile + rg - 1) / rg, c->cu_count);
+        const int64_t items = (int64_t)((ntile + rg * grid - 1) / (rg * grid)) * ((ns + kg - 1) / kg);
+        if (items < best) {
+            best = items;
+            m.kg = kg;
+            p.grid = grid;
+        }
+    }
+    return p;
+}
+}  // namespace
 // nv_tail: vectors of the last blockIdx.y slice when it differs from B (the second group of a
 // 5..7-vector call)
 static int gemv_impl(int ty, const void *W, int64_t row_stride, int K, int rows, const float *x, int64_t x_stride,
@@ -430,33 +503,29 @@ static int gemv_impl(int ty, const void *W, int64_t row_stride, int K, int rows,
         a.accumulate = accumulate;
         return stream_any(0, ty, a, n_batch, (hipStream_t)s);
     }
-    // Vectors of Q8_0 / Q4_K / Q5_K / Q6_K in one pass on int8 MFMA, every weight read once for all
-    // vectors (gs_k_mv_<ty>_<0|1>: 16 rows per workgroup, the row in chunks of up to 4096 elements
-    // in LDS with the vectors' q8_1 units). Rows: whole chunks of whole 16-byte pieces, 16-byte
-    // aligned rows and activations. Taken where it beats the streaming kernels (measured, one
-    // MI355X, 4096 x 4096, 12288 x 4096, 4096 x 12288): from 5 vectors, where they read the
-    // matrix twice (Q4_K 12288 x 4096 x 8 vectors: 20.2 against 24.5 us, Q8_0 19.6 against 25.2),
-    // from 3 when rows are longer than their register plan (K > 4096: one vector per slice; Q6_K
-    // 4096 x 12288 x 4 vectors: 26.4 against 30.3 us), and for Q8_0 from 3 (4096 x 4096: 7.8 against
-    // 8.5 us at 3 vectors, 7.9 against 9.2 at 4); below that they stay faster (they overlap the dot
-    // products with the weight stream, where this kernel waits for a tile's bytes).
-    const int mv_min = ty == GS_Q8_0 || K > 4096 ? 3 : 5;
-    if ((ty == GS_Q8_0 || ty == GS_Q4_K || ty == GS_Q5_K || ty == GS_Q6_K) && B >= mv_min && n_batch == 1 && nv_tail == 0 &&
-        aligned16(x) && x_stride % 4 == 0 && aligned16(W) && row_stride % 16 == 0) {
-        const int ck = std::min(K, 4096);
-        const int64_t rbytes = (int64_t)(ck / qk) * bb;
-        if (K % ck == 0 && ck % qk == 0 && rbytes % 16 == 0 && rbytes <= 4352) {
-            MvArgs m{(const uint8_t *)W, row_stride, x, x_stride, y, y_stride, K, rows, B, accumulate};
-            const size_t U = ck / 32, lds = 16 * ((size_t)rbytes + 16) + 320 * U + 8 * 64 * 16;
-            // one workgroup per CU at most (its LDS), each walking tiles of 16 rows
-            hipError_t e;
-            DeviceCtx *c = ctx(&e);
-            if (!c) return e;
-            const int ntile = (rows + 15) / 16, grid = std::min(ntile, c->cu_count);
+    if (n_batch == 1 && nv_tail == 0 && B >= mv_min(ty, K, rows)) {
+        hipError_t e;
+        DeviceCtx *c = ctx(&e);
+        if (!c) return e;
+        MvArgs m{(const uint8_t *)W, row_stride, x, x_stride, y, y_stride, K, rows, B, accumulate, 0, 0, 0};
+        // the workgroup form (measured beside it): Q8_0 rows in one chunk, or of more than 8192 elements
+        // with 5..8 vectors (4096 x 12288 x 8: 24.3 us against 25.1; 4 vectors 20.8 against 18.3), and
+        // Q6_K with 5..8 vectors on one tile of 16 rows per CU
+        const int ck = std::min(K, 4096), ntile = (rows + 15) / 16, grid = std::min(ntile, c->cu_count);
+        const bool q8 = ty == GS_Q8_0 && (K <= 4096 || (K > 8192 && B > 4));
+        const bool q6 = ty == GS_Q6_K && K <= 4096 && B > 4 && ntile <= grid;
+        if ((q8 || q6) && aligned16(x) && x_stride % 4 == 0 && aligned16(W) && row_stride % 16 == 0 && K % ck == 0 &&
+            ck % 256 == 0 && (ck / qk * bb) % 16 == 0) {
+            const size_t U = ck / 32, lds = 16 * ((size_t)ck / qk * bb + 16) + 288 * U + 8 * 64 * 16;
             const bool multi = ntile > grid || K > ck;
-            return launch("gs_k_mv_" + std::to_string(ty) + (multi ? "_1" : "_0"), dim3((unsigned)grid), dim3(512), lds,
+            return launch(std::string("gs_k_mvc_") + (q8 ? multi ? "8_1" : "8_0" : "14_0"), dim3((unsigned)grid), dim3(512), lds,
                           (hipStream_t)s, m);
         }
+        // (Q8_0 rows of one chunk off 16-byte boundaries, 3 or 4 vectors: streamed, 7.5 us against 8.5)
+        const MvPlan p = ty == GS_Q8_0 && K <= 4096 && B <= 4 ? MvPlan() : mv_plan(c, ty, m);
+        if (p.depth)
+            return launch("gs_k_mv_" + std::to_string(ty) + "_" + std::to_string(B <= 4 ? 1 : 2) + "_" + std::to_string(p.depth),
+                          dim3((unsigned)p.grid), dim3(512), p.lds, (hipStream_t)s, m);
     }
     // more than 4 vectors whose units do not fit 8-vector registers (K > 2048): groups of 4 vectors
     // over the whole K instead of K slices of 8 vectors (8 x 4096 Q8_0: 14 us against 28 us), both
@@ -859,18 +928,6 @@ struct QgShape {
     int slices;               // K slices (blockIdx.z), partial tiles in the workspace
     double us;                // modelled time
 };
-struct QgFmt {
-    int slot, table;          // bytes of a super-block's LDS slot and of the decode tables
-    bool dwords;              // rows start on dwords (formats whose super-block is whole dwords)
-    double cost;              // decode cost against Q4_K, from measured calls
-};
-const QgFmt *qg_fmt(int ty) {
-    static const std::map<int, QgFmt> f = {{GS_Q8_0, {272, 0, true, 1.15}},     {GS_Q4_K, {144, 0, true, 1.0}},
-                                           {GS_Q5_K, {176, 0, true, 1.1}},      {GS_Q6_K, {240, 0, false, 1.25}},
-                                           {GS_IQ2_XXS, {80, 5120, false, 1.15}}, {GS_IQ3_XXS, {112, 3072, false, 1.3}}};
-    const auto it = f.find(ty);
-    return it == f.end() ? nullptr : &it->second;
-}
 // LDS of a kernel: tables, the activation buffers, two buffers of the raw chunk; at least the partial
 // tiles of the end (qgemm.hip has the same figures)
 size_t qg_lds(const QgFmt &f, const QgShape &q) {

@@ -71,7 +71,7 @@ struct QuantArgs {
     int64_t n_blocks;
 };
 
-// multi-vector Q8_0 GEMV on int8 MFMA (gs_gemv with 2..8 vectors): y[t][r] (+)= W[r] . q8_1(x[t])
+// GEMV of 2..8 vectors on int8 MFMA (mvgemv.hip): y[t][r] (+)= W[r] . q8_1(x[t])
 struct MvArgs {
     const uint8_t *w;
     int64_t row_stride;   // bytes
@@ -80,6 +80,8 @@ struct MvArgs {
     float *y;
     int64_t y_stride;     // floats
     int K, rows, nv, accumulate;
+    int ck, nchunk;       // elements per chunk of K (a multiple of 256), chunks
+    int kg;               // waves along K (1, 2, 4, 8); 8 / kg row tiles side by side
 };
 
 // f32 rows -> compact f16 rows (round to nearest even): N rows of K values, source row stride

@@ -37,12 +37,12 @@
 #include <stdint.h>
 #include "kargs.h"
 #include "formats.h"
+#include "lds_load.h"
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 #define QG_TH 512
 #define QG_WV 8
@@ -71,14 +71,6 @@ __device__ __forceinline__ uint32_t lw32(const uint8_t *p) { return *(const uint
 __device__ __forceinline__ uint2 lw64(const uint8_t *p) { return *(const uint2 *)p; }
 
 #define QG_2P24 16777216.0f
-// a wave-uniform pointer whose 64-bit arithmetic ran on the vector unit, back in scalar registers
-// (a buffer resource or scalar base kept in VGPRs costs a readfirstlane loop per load)
-__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *p) {
-    const uint64_t v = (uint64_t)p;
-    return (const uint8_t *)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32) |
-                             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v));
-}
-
 // 8 bytes at LDS offset p + sh (p dword-aligned, sh 0 or 2): three dwords shifted into place
 struct W3 { uint32_t a, b, c; };
 __device__ __forceinline__ W3 lw3(const uint8_t *p) { return W3{lw32(p), lw32(p + 4), lw32(p + 8)}; }
@@ -271,25 +263,6 @@ struct QgIQ3 {   // lib.rs:312-328
         return iq_mix8(make_uint4(r.a.x, r.a.y, r.b.x, r.b.y), r.sm, p.D);
     }
 };
-
-// 16 bytes per lane from rsrc + voff + soff to LDS address lds + 16 lane, in flight on the vector-memory
-// counter. Written as an asm statement because the compiler waits for every outstanding load of this
-// kind before any LDS read; the waits are placed by hand (wait_vm) instead. No register is written but
-// M0, which the compiler only holds between a write of its own and the instruction that needs it.
-__device__ __forceinline__ void dma16(uint32_t lds, uint32_t voff, uint32_t soff, u4 rsrc) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff), "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff)) : "memory");
-}
-// the words of a raw buffer resource over `bytes` bytes from a wave-uniform base (as BufferAt makes it)
-__device__ __forceinline__ u4 rsrc_words(const uint8_t *base, uint32_t bytes) {
-    const uint64_t b = (uint64_t)base;
-    return u4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, bytes, 0x00020000u};
-}
-template <int N>
-__device__ __forceinline__ void wait_vm() {   // until at most N vector-memory operations are outstanding
-    static_assert(N < 64, "vmcnt");
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory");
-}
 
 // XH: the activations come as f16 half-slabs from the workspace (gs_k_qgemm_x), else f32 rows.
 template <class F, int NR, int NT, int RG, int KG, int RC, bool XH>
