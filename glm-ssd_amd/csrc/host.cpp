@@ -125,13 +125,15 @@ hipError_t get_fn(DeviceCtx *c, const std::string &name, hipFunction_t *f) {
         *f = it->second;
         return hipSuccess;
     }
+    const hipError_t pending = hipPeekAtLastError();
     for (hipModule_t m : c->mods) {
-        if (hipModuleGetFunction(f, m, name.c_str()) == hipSuccess) {
+        const bool hit = hipModuleGetFunction(f, m, name.c_str()) == hipSuccess;
+        if (!hit && pending == hipSuccess) (void)hipGetLastError();   // a miss is no error of the caller's
+        if (hit) {
             c->fns[name] = *f;
             return hipSuccess;
         }
     }
-    (void)hipGetLastError();  // clear the lookup misses
     fprintf(stderr, "glmssd: kernel %s not found in the embedded code objects\n", name.c_str());
     return hipErrorNotFound;
 }

@@ -6,7 +6,7 @@ import os
 
 import numpy as np
 
-from . import DeviceBuffer, ExpertPtrs, ops
+from . import DeviceBuffer, Event, ExpertPtrs, MoeBatch, check, lib, ops
 from .types import GgmlType as T, row_bytes
 
 
@@ -112,14 +112,39 @@ def route(logits, bias, k, weights_norm=True, weights_scale=1.0):
     scores + 1e-20) * scale (the sum is 1 without normalisation). logits: [t][n_expert] f32."""
     logits = np.asarray(logits, dtype=np.float32)
     bias = np.asarray(bias, dtype=np.float32)
-    out = []
-    for row in logits.reshape(-1, bias.size):
-        scores = (1.0 / (1.0 + np.exp(-row.astype(np.float32)))).astype(np.float32)
-        sel = scores + bias
-        order = sorted(range(bias.size), key=lambda e: -sel[e])[:k]   # stable: ties keep id order
-        wsum = np.float32(sum(scores[e] for e in order)) if weights_norm else np.float32(1.0)
-        out.append([(e, float(scores[e] / (wsum + np.float32(1e-20)) * np.float32(weights_scale))) for e in order])
-    return out
+    scores = (1.0 / (1.0 + np.exp(-logits.reshape(-1, bias.size)))).astype(np.float32)
+    order = np.argsort(-(scores + bias), axis=1, kind="stable")[:, :k]   # ties keep id order
+    chosen = np.take_along_axis(scores, order, axis=1)
+    wsum = np.full((len(scores), 1), 0.0 if weights_norm else 1.0, np.float32)
+    if weights_norm:
+        for i in range(chosen.shape[1]):   # in rank order, in float32
+            wsum += chosen[:, i:i + 1]
+    w = chosen / (wsum + np.float32(1e-20)) * np.float32(weights_scale)
+    return [list(zip(e, v)) for e, v in zip(order.tolist(), w.tolist())]
+
+
+class _PinnedF32:
+    """Page-locked host floats that a stream copies device values into, and the event of the last copy."""
+
+    def __init__(self, n):
+        self.p, self.done = C.c_void_p(), Event(timed=False)
+        check(lib().gs_host_alloc(C.byref(self.p), 4 * n))
+        self.a = np.ctypeslib.as_array(C.cast(self.p, C.POINTER(C.c_float)), (n,))
+
+    def start(self, src, n, s):
+        check(lib().gs_memcpy_d2h(self.p, src.p, 4 * n, s.raw() if s else None))
+        check(lib().gs_event_record(self.done.h, s.raw() if s else None))
+
+    def wait(self, n):
+        self.done.sync()
+        return self.a[:n]
+
+    def __del__(self):
+        try:
+            if self.p:
+                lib().gs_host_free(self.p)
+        except Exception:
+            pass
 
 
 class Mat:
@@ -133,6 +158,9 @@ class Mat:
 
     def ptr(self):
         return self.buf.ptr(self.offset)
+
+    def address(self):
+        return self.buf.p.value + self.offset
 
 
 class MoeLayer:
@@ -152,11 +180,11 @@ class MoeLayer:
     1071-1081); multi-token paths write every (route rank, token) pair into its own slot and sum
     the slots in rank order (forward.rs:1119-1127), so the output is bit-reproducible."""
     MOE_MAX, PER_TOKEN_MAX = 16, 16
+    LOGITS_MAX = 64   # tokens whose logits the layer's page-locked buffer holds
 
     def __init__(self, router, bias, shared, experts, n_embd, n_ff, ty_gu, ty_down, k=8, weights_norm=True,
                  weights_scale=1.0, clamp_exp=0.0, clamp_shexp=0.0, router_ty=T.F32, shared_ty=(T.Q6_K,) * 3,
                  n_ff_shexp=None, s=None, deterministic=None):
-        from . import MoeBatch   # noqa: F401  (layout shared with the C ABI)
         self.n_embd, self.n_ff, self.k = n_embd, n_ff, k
         self.deterministic = deterministic_default() if deterministic is None else bool(deterministic)
         self.n_exp = len(experts)
@@ -177,12 +205,24 @@ class MoeLayer:
             self.grouped = ResidentMoeLayer([e[0] for e in experts], [e[1] for e in experts],
                                             [e[2] for e in experts], n_embd, n_ff, ty_gu, ty_down)
         self._scratch = {}
+        self._logits = _PinnedF32(self.LOGITS_MAX * self.n_exp)
         self.last_routes = None
 
     def _buf(self, name, nbytes):
         b = self._scratch.get(name)
         if b is None or b.nbytes < nbytes:
             b = self._scratch[name] = DeviceBuffer(max(nbytes, 4))
+        return b
+
+    def _batch(self, r):
+        """MoeBatch of one token over the (expert, weight) pairs r"""
+        b = MoeBatch()
+        b.n = n = len(r)
+        ids = [e for e, _ in r]
+        b.gate[:n] = [self.gate[e].address() for e in ids]
+        b.up[:n] = [self.up[e].address() for e in ids]
+        b.down[:n] = [self.down[e].address() for e in ids]
+        b.w[0][:n] = [w for _, w in r]
         return b
 
     def _mm(self, m, x, y, t, s, x_stride=None, y_stride=None):
@@ -202,13 +242,16 @@ class MoeLayer:
     def forward(self, xn, out, t, s=None):
         """xn: device [t][n_embd] (normalised hidden states); out: device [t][n_embd], overwritten
         with shared-expert FFN + routed-expert FFN. Returns the routes."""
-        from . import MoeBatch
         n, ne = self.n_embd, self.n_exp
         logits_d = self._buf("logits", t * ne * 4)
         self._mm(self.router, xn, logits_d, t, s)
-        logits = logits_d.download(np.float32, t * ne, s)
-        routes = route(logits.reshape(t, ne), self.bias, self.k, self.norm, self.scale)
-        self.last_routes = routes
+        # up to LOGITS_MAX tokens the shared expert is launched before the host waits for the logits and
+        # routes, so the GPU works meanwhile (4 tokens, 32 experts of 512 x 2048, with the routing in
+        # whole-array steps: 162 -> 83 us a layer)
+        if t <= self.LOGITS_MAX:
+            self._logits.start(logits_d, t * ne, s)
+        else:
+            logits = logits_d.download(np.float32, t * ne, s)
         # shared expert (forward.rs:1108-1110, swiglu_ffn :915-921)
         g, u = self._buf("sh_g", t * self.n_ff_sh * 4), self._buf("sh_u", t * self.n_ff_sh * 4)
         self._mm(self.sh[0], xn, g, t, s)
@@ -217,11 +260,10 @@ class MoeLayer:
         self._mm(self.sh[2], g, out, t, s)
         acc = self._buf("acc", t * n * 4)
         acc.zero(s)
-        groups = [[] for _ in range(ne)]
-        for ti, r in enumerate(routes):
-            for e, w in r:
-                groups[e].append((ti, w))
-        used = [e for e in range(ne) if groups[e]]
+        if t <= self.LOGITS_MAX:
+            logits = self._logits.wait(t * ne)
+        routes = route(logits.reshape(t, ne), self.bias, self.k, self.norm, self.scale)
+        self.last_routes = routes
         if t <= self.PER_TOKEN_MAX:
             # decode, MTP and short-batch sizes: a one-token FFN per token over its own experts, the
             # tokens in gs_moe_ffn_tokens calls of up to 32 (token, expert) pairs when their expert
@@ -233,15 +275,7 @@ class MoeLayer:
                 per = max(1, 32 // kk)
                 h = self._buf("h", min(t, per) * kk * self.n_ff * 4)
                 for t0 in range(0, t, per):
-                    bs = []
-                    for r in routes_d[t0:t0 + per]:
-                        b = MoeBatch()
-                        b.n = kk
-                        for i, (e, w) in enumerate(r):
-                            b.gate[i], b.up[i], b.down[i] = (self.gate[e].ptr().value, self.up[e].ptr().value,
-                                                             self.down[e].ptr().value)
-                            b.w[0][i] = w
-                        bs.append(b)
+                    bs = [self._batch(r) for r in routes_d[t0:t0 + per]]
                     ops.moe_ffn_tokens(self.ty_gu, self.ty_down, bs, self.gate[0].row_bytes, n, self.n_ff,
                                        self.down[0].row_bytes, _at(xn, t0 * n * 4), h, acc.ptr(t0 * n * 4),
                                        self.lim, s)
@@ -249,13 +283,7 @@ class MoeLayer:
             h = self._buf("h", self.MOE_MAX * self.n_ff * 4)
             for ti, r in enumerate(routes_d):
                 for b0 in range(0, len(r), self.MOE_MAX):
-                    chunk = r[b0:b0 + self.MOE_MAX]
-                    b = MoeBatch()
-                    b.n = len(chunk)
-                    for i, (e, w) in enumerate(chunk):
-                        b.gate[i], b.up[i], b.down[i] = (self.gate[e].ptr().value, self.up[e].ptr().value,
-                                                         self.down[e].ptr().value)
-                        b.w[0][i] = w
+                    b = self._batch(r[b0:b0 + self.MOE_MAX])
                     ops.moe_ffn(self.ty_gu, self.ty_down, b, 1, self.gate[0].row_bytes, n, self.n_ff,
                                 self.down[0].row_bytes, _at(xn, ti * n * 4), h, acc.ptr(ti * n * 4), self.lim, s)
         elif self.grouped is not None:
@@ -269,6 +297,11 @@ class MoeLayer:
                 self.grouped.forward(xn, acc, t, self.lim, s)
         else:
             # run_expert_rows (forward.rs:1399-1413) per used expert
+            groups = [[] for _ in range(ne)]
+            for ti, r in enumerate(routes):
+                for e, w in r:
+                    groups[e].append((ti, w))
+            used = [e for e in range(ne) if groups[e]]
             offs, idx, w, pe = group_pairs(routes, ne)
             d_idx, d_w = DeviceBuffer.from_array(idx, s), DeviceBuffer.from_array(w, s)
             to, slots = d_idx, None
