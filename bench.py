@@ -307,7 +307,7 @@ def run_gemm(L, s, ty, rows, K, N, make, steps, warmup, seed, min_rot_bytes=640 
             "weight_GBps": round(raw.nbytes / t / 1e9, 1), "tokens": N, "rotated_copies": n}
 
 
-GROUPED_KERNELS = ("gs_k_grouped_16_1_2_2_8", "gs_k_grouped_16_2_2_4_8")   # config 5's gate/up and down
+GROUPED_KERNELS = ("gs_k_grouped_16_1", "gs_k_grouped_16_2")   # config 5's gate/up and down
 
 
 def config5_roofline(r):

@@ -23,6 +23,7 @@
 // routing-weighted result into y[token] with f32 atomics (the combine of quants.cu:324-363).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 #include "kargs.h"
 #include "formats.h"
 
@@ -112,13 +113,23 @@ struct FragRaw {
     uint2 sm;
     uint2 g2;   // IQ3_XXS: the second 4-value entry
 };
+// A constant in a scalar register that the compiler does not look through: the address arithmetic of the
+// contraction's two copies is otherwise hoisted in front of the branch that picks one, every
+// fragment's at once (50 registers).
+__device__ __forceinline__ uint32_t opaque(uint32_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
 template <int G>
 __device__ __forceinline__ uint32_t sign_off(uint32_t a1, uint32_t r16) {
-    return (__builtin_amdgcn_ubfe(a1, 7 * G, 7) << 7) | r16;
+    // the field moved to bits 7..13, masked and merged by one v_bitop3 (shift and bitop3 issue in half the
+    // time of v_bfe and v_lshl_or)
+    const uint32_t t = G == 0 ? a1 << opaque(7) : a1 >> (G == 1 ? 0 : opaque(7 * (G - 1)));
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)t, 0x3f80, (int)r16, 0xEA);   // (t & m) | r16
 }
 template <int G>
 __device__ __forceinline__ void iq2_frag_fetch(const uint8_t *tab, uint32_t a0, uint32_t a1, uint32_t r16, FragRaw &r) {
-    const uint32_t ga = __builtin_amdgcn_perm(a0, a1 & 0xF0000000u, 0x0c0c0403u + (G << 8));
+    const uint32_t ga = __builtin_amdgcn_perm(a0, a1 & 0xF0000000u, opaque(0x0c0c0403u + (G << 8)));
     r.g = *(const uint4 *)(tab + GS_GRP_GRID_OFF + ga);
     r.sm = *(const uint2 *)(tab + sign_off<G>(a1, r16));
 }
@@ -128,8 +139,8 @@ __device__ __forceinline__ void iq3_frag_fetch(const uint8_t *tab, uint32_t g0, 
     const uint32_t gw = G < 2 ? g0 : g1;
     constexpr uint32_t b0 = (2 * G) & 3;
     const uint32_t hs = a1 & 0xF0000000u;
-    const uint2 lo = *(const uint2 *)(tab + GS_GRP_GRID_OFF + __builtin_amdgcn_perm(gw, hs, 0x0c0c0403u + (b0 << 8)));
-    r.g2 = *(const uint2 *)(tab + GS_GRP_GRID_OFF + __builtin_amdgcn_perm(gw, hs, 0x0c0c0403u + ((b0 + 1) << 8)));
+    const uint2 lo = *(const uint2 *)(tab + GS_GRP_GRID_OFF + __builtin_amdgcn_perm(gw, hs, opaque(0x0c0c0403u + (b0 << 8))));
+    r.g2 = *(const uint2 *)(tab + GS_GRP_GRID_OFF + __builtin_amdgcn_perm(gw, hs, opaque(0x0c0c0403u + ((b0 + 1) << 8))));
     r.g = make_uint4(lo.x, lo.y, 0u, 0u);
     r.sm = *(const uint2 *)(tab + sign_off<G>(a1, r16));
 }
@@ -148,7 +159,14 @@ __device__ __forceinline__ h8 frag_finish(const FragRaw &r) {
                                              g.w ^ ((r.sm.y << 1) & M)));
 }
 
-#define GS_GRP_AV_LOAD(tt, cc) __builtin_bit_cast(h8, *(const uint4 *)(slab + (16 * (tt) + j) * 512 + ((((cc) ^ j)) << 4)))
+// f(integral_constant<int, I>) for I in [A, B)
+template <int A, int B, class Fn>
+__device__ __forceinline__ void static_for(Fn &&f) {
+    if constexpr (A < B) {
+        f(std::integral_constant<int, A>());
+        static_for<A + 1, B>(f);
+    }
+}
 
 __device__ __forceinline__ float grp_swiglu(float g, float u, float lim) {   // ops.cu:101-115
     if (lim > 0.f) {
@@ -163,12 +181,9 @@ __device__ __forceinline__ float grp_swiglu(float g, float u, float lim) {   // 
 // side by side. (Scheduling experts by pair count, largest first, made no difference at 512
 // tokens: every tile streams the same K, so tiles cost about the same; the count ranking itself,
 // done by every workgroup, took 10 us of a 4-token call.)
-// m_tmp: n_exp ints of scratch (the staging area, free during the prologue).
-template <int NTH>
-__device__ __forceinline__ void grp_prefix(const GroupedArgs &a, int MT, int nrb, int *m_tmp, int *pre) {
+// m_tmp: the experts' pair counts (the staging area, free during the prologue).
+__device__ __forceinline__ void grp_prefix(const GroupedArgs &a, int MT, int nrb, const int *m_tmp, int *pre) {
     const int tid = threadIdx.x, lane = tid & 63;
-    for (int e = tid; e < a.n_exp; e += NTH) m_tmp[e] = a.offs[e + 1] - a.offs[e];
-    __syncthreads();
     if (tid < 64) {
         int carry = 0;
         for (int r0 = 0; r0 < a.n_exp; r0 += 64) {
@@ -222,15 +237,15 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs &a) {
         (uint8_t *)__builtin_bit_cast(__attribute__((address_space(3))) uint8_t *, (uint32_t)0);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = lane & 15, q = lane >> 4;
+    const uint32_t xlane = 512u * j + (uint32_t)(((8 * q) ^ j) << 4);   // the lane's chunk 8q of its token slot
     const uint32_t r16 = (uint32_t)j << 3;   // the lane's sign-table replica
     const int K = a.K, rows = a.rows, nsb = K / 256;
     const int nrb = (rows + RB - 1) / RB;
     const uint32_t rs = (uint32_t)a.row_stride;
     uint8_t *const tab = gs_grp_dyn;
     uint8_t *const stage = gs_grp_dyn + GS_GRP_TAB_BYTES;
-    grp_tables<TY, NTH>(tab, tid);
     GrpMeta &M = *(GrpMeta *)(gs_grp_dyn + GS_GRP_TAB_BYTES + 4 * SLAB);
-    grp_prefix<NTH>(a, MT, nrb, (int *)stage, M.pre);
+    grp_prefix(a, MT, nrb, (const int *)stage, M.pre);
     __syncthreads();
     const int total = M.pre[a.n_exp];
     // Workgroup w runs on XCD w % 8 (round-robin dispatch). With a grid that is a multiple of 8,
@@ -425,6 +440,55 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs &a) {
     auto wait_slot = [&]() __attribute__((always_inline)) {
         if (pos > 1) wait_count(&M.cnt[buf], (uint32_t)(NTH / 64) * (pos / 4u + 1u));
     };
+    // One position: the 8 x NR x MATS fragments of the wave's rows in order, the table reads of fragment
+    // f + DEP issued before fragment f is finished and multiplied (an LDS read takes as long as about
+    // three fragments' arithmetic, and two waves per SIMD hide little of it), the activations of the
+    // next MFMA column likewise; before, each column's four fragments were read, awaited and then
+    // multiplied (512 tokens to 288 experts 713 -> 693 us, 2048 1449 -> 1395). NL: the tile's live token
+    // sub-tiles (one, or all). The scheduling barrier keeps the order where the compiler would spill.
+    auto contract = [&](auto live, const WRegs &wu, uint32_t xa) __attribute__((always_inline)) {
+        constexpr int NL = decltype(live)::value, NB = NR * MATS, NF = 8 * NB, 
+                      DEP = IQ3 ? (KIND == 1 && NT * NR == 4 ? 1 : 2) : 3;   // as far as the registers allow
+        f4 sb[NL][NR][MATS];
+#pragma unroll
+        for (int tt = 0; tt < NL; tt++)
+#pragma unroll
+            for (int n = 0; n < NR; n++)
+#pragma unroll
+                for (int mt = 0; mt < MATS; mt++) sb[tt][n][mt] = f4{0.f, 0.f, 0.f, 0.f};
+        FragRaw fr[DEP + 1];
+        h8 av[2][NL];
+        auto fetch = [&](auto fi) __attribute__((always_inline)) {
+            constexpr int f = decltype(fi)::value, m = f / NB, G = m & 3, n = f % NB / MATS, mt = f % MATS;
+            const uint4 w = wu.q[n][mt];
+            if constexpr (IQ3) iq3_frag_fetch<G>(tab, m < 4 ? w.x : w.z, m < 4 ? w.y : w.w, m < 4 ? wu.sg[n][mt].x : wu.sg[n][mt].y, r16, fr[f % (DEP + 1)]);
+            else iq2_frag_fetch<G>(tab, m < 4 ? w.x : w.z, m < 4 ? w.y : w.w, r16, fr[f % (DEP + 1)]);
+        };
+        auto load_av = [&](auto mi) __attribute__((always_inline)) {
+            constexpr int m = decltype(mi)::value;
+#pragma unroll
+            for (int tt = 0; tt < NL; tt++) av[m & 1][tt] = __builtin_bit_cast(h8, *(const uint4 *)(gs_grp_dyn + (xa ^ (m << 4)) + 8192 * tt));
+        };
+        static_for<0, DEP>(fetch);
+        load_av(std::integral_constant<int, 0>());
+        static_for<0, NF>([&](auto fi) __attribute__((always_inline)) {
+            constexpr int f = decltype(fi)::value, m = f / NB, n = f % NB / MATS, mt = f % MATS;
+            if constexpr (f + DEP < NF) fetch(std::integral_constant<int, f + DEP>());
+            if constexpr (f % NB == 0 && m < 7) load_av(std::integral_constant<int, m + 1>());
+            if constexpr (NL > 1 || (NT > 1 && !(IQ3 && KIND == 1))) __builtin_amdgcn_sched_barrier(0);
+            const h8 bf = frag_finish<IQ3>(fr[f % (DEP + 1)]);
+#pragma unroll
+            for (int tt = 0; tt < NL; tt++) sb[tt][n][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[m & 1][tt], bf, sb[tt][n][mt], 0, 0, 0);
+        });
+#pragma unroll
+        for (int n = 0; n < NR; n++)
+#pragma unroll
+            for (int mt = 0; mt < MATS; mt++) {
+                const float cd = h2f((uint32_t)__builtin_amdgcn_ds_bpermute((j + 16 * (n * MATS + mt)) << 2, (int)wu.dq)) * XS;
+#pragma unroll
+                for (int tt = 0; tt < NL; tt++) acc[tt][n][mt] += cd * sb[tt][n][mt];
+            }
+    };
     auto step = [&](WRegs &wu, WRegs &wl) __attribute__((always_inline)) -> bool {
         wait_slot();
         // Issue priority follows the lag: every wave stores its share of each slot, so the
@@ -464,52 +528,10 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs &a) {
 
         // ---- contract position (cur, b) ------------------------------------------------------
         {
-            const uint8_t *slab = stage + buf * SLAB;
-            const int n_here = cur.n_here;
-            f4 sb[NT][NR][MATS];
-#pragma unroll
-            for (int tt = 0; tt < NT; tt++)
-#pragma unroll
-                for (int n = 0; n < NR; n++)
-#pragma unroll
-                    for (int mt = 0; mt < MATS; mt++) sb[tt][n][mt] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int hu = 0; hu < 2; hu++) {    // unit 2q + hu
-#define GS_GRP_FRAGS(G)                                                                            \
-        FragRaw fr[NR][MATS];                                                                      \
-        _Pragma("unroll") for (int n = 0; n < NR; n++)                                             \
-        _Pragma("unroll") for (int mt = 0; mt < MATS; mt++) {                                      \
-            if (IQ3) iq3_frag_fetch<G>(tab, hu ? wu.q[n][mt].z : wu.q[n][mt].x, hu ? wu.q[n][mt].w : wu.q[n][mt].y, \
-                                       hu ? wu.sg[n][mt].y : wu.sg[n][mt].x, r16, fr[n][mt]);       \
-            else iq2_frag_fetch<G>(tab, hu ? wu.q[n][mt].z : wu.q[n][mt].x, hu ? wu.q[n][mt].w : wu.q[n][mt].y, r16, fr[n][mt]); \
-        }                                                                                          \
-        _Pragma("unroll") for (int n = 0; n < NR; n++)                                             \
-        _Pragma("unroll") for (int mt = 0; mt < MATS; mt++) bf[n][mt] = frag_finish<IQ3>(fr[n][mt]);
-#define GS_GRP_STEP(G)                                                                             \
-    {                                                                                              \
-        h8 bf[NR][MATS];                                                                           \
-        GS_GRP_FRAGS(G)                                                                            \
-        const int cc = 8 * q + 4 * hu + G;                                                         \
-        _Pragma("unroll") for (int tt = 0; tt < NT; tt++)                                          \
-            if (tt == 0 || 16 * tt < n_here) {                                                     \
-                const h8 av = GS_GRP_AV_LOAD(tt, cc);                                              \
-                _Pragma("unroll") for (int n = 0; n < NR; n++)                                     \
-                _Pragma("unroll") for (int mt = 0; mt < MATS; mt++)                                \
-                    sb[tt][n][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bf[n][mt], sb[tt][n][mt], 0, 0, 0);                     \
-            }                                                                                      \
-    }
-                GS_GRP_STEP(0) GS_GRP_STEP(1) GS_GRP_STEP(2) GS_GRP_STEP(3)
-#undef GS_GRP_STEP
-            }
-#pragma unroll
-            for (int n = 0; n < NR; n++)
-#pragma unroll
-                for (int mt = 0; mt < MATS; mt++) {
-                    const float cd = h2f((uint32_t)__builtin_amdgcn_ds_bpermute((j + 16 * (n * MATS + mt)) << 2, (int)wu.dq)) * XS;
-#pragma unroll
-                    for (int tt = 0; tt < NT; tt++)
-                        if (tt == 0 || 16 * tt < n_here) acc[tt][n][mt] += cd * sb[tt][n][mt];
-                }
+            // chunk 8q + m of token slot j lies at chunk position (8q + m) ^ j = (8q ^ j) ^ m
+            const uint32_t xa = GS_GRP_TAB_BYTES + (uint32_t)buf * SLAB + xlane;
+            if (NT > 1 && cur.n_here > 16) contract(std::integral_constant<int, NT>(), wu, xa);
+            else contract(std::integral_constant<int, 1>(), wu, xa);
         }
 
         // ---- tile epilogue: lane holds tokens 16t + 4q + i (i < 4) of row row0 + 16n + j ----
@@ -592,28 +614,79 @@ __device__ __forceinline__ void grouped_body(const GroupedArgs &a) {
     }
 }
 
+// the kernels' common start: decode tables and pair counts into LDS
+template <int TY, int NTH>
+__device__ __forceinline__ int *grp_start(const GroupedArgs &a) {
+    uint8_t *const lds =
+        (uint8_t *)__builtin_bit_cast(__attribute__((address_space(3))) uint8_t *, (uint32_t)0);
+    int *const m_tmp = (int *)(lds + GS_GRP_TAB_BYTES);
+    // the first counts' loads are in flight while the tables are built
+    const int tid = threadIdx.x, e0 = min(tid, a.n_exp - 1);
+    const int o0 = a.offs[e0], o1 = a.offs[e0 + 1];
+    grp_tables<TY, NTH>(lds, tid);
+    if (tid < a.n_exp) m_tmp[tid] = o1 - o0;
+    for (int e = tid + NTH; e < a.n_exp; e += NTH) m_tmp[e] = a.offs[e + 1] - a.offs[e];
+    __syncthreads();
+    return m_tmp;
+}
+
+// Prompts (more than 64 pairs): the tile shape with the least work, chosen by every workgroup alike from
+// the pair counts, which only the device knows: rounds of the persistent grid times a tile's cost. A
+// tile of half the rows costs about half (of a round of the largest, fitted over 17..400 tokens to 288 experts
+// of 1536 x 4096 and 96 of 2048 x 4096: gate/up 2x1 0.57, 1x1 0.52; down 2x2 0.55, 1x2 0.51, IQ3_XXS
+// 0.48, 0.43), so what decides is the last round and how many chunks of 32 or 16 pairs the routing
+// makes. 37 tokens to 96 experts, 76 used: 286 us with 3 + 3 rounds of the largest tiles, 241 with 5 + 5 of half
+// ones; 512 tokens to 288 keep the largest (1x1 and 1x2 tiles: 12 % slower). The three shapes are one
+// kernel because the choice needs the counts.
+template <int TY, int KIND>
+__device__ __forceinline__ void grouped_auto(const GroupedArgs &a) {
+    const int *m_tmp = grp_start<TY, 512>(a);
+    int n16 = 0, n32 = 0;
+    for (int e = threadIdx.x & 63; e < a.n_exp; e += 64) {
+        const int m = max(m_tmp[e], 0);
+        n16 += (m + 15) >> 4;
+        n32 += (m + 31) >> 5;
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        n16 += __shfl_xor(n16, o);
+        n32 += __shfl_xor(n32, o);
+    }
+    n16 = __builtin_amdgcn_readfirstlane(n16);
+    n32 = __builtin_amdgcn_readfirstlane(n32);
+    constexpr int RB = KIND == 1 ? 256 : 512;   // rows of the largest shape's tile; the others take half
+    const int g = gridDim.x, nb = (a.rows + RB - 1) / RB, nb2 = (a.rows + RB / 2 - 1) / (RB / 2);
+    constexpr int C0 = 100, C1 = KIND == 1 ? 57 : TY == GS_IQ3_XXS ? 48 : 55,
+                  C2 = KIND == 1 ? 52 : TY == GS_IQ3_XXS ? 43 : 51;
+    const int c0 = (n32 * nb + g - 1) / g * C0, c1 = (n32 * nb2 + g - 1) / g * C1, c2 = (n16 * nb2 + g - 1) / g * C2;
+    // (IQ3_XXS down: two of the middle shape's rounds cost less than one of the largest's, never more of them)
+    constexpr bool ALL = KIND == 1 || TY != GS_IQ3_XXS;
+    if (ALL && c0 <= c1 && c0 <= c2) grouped_body<TY, KIND, 2, KIND == 1 || !ALL ? 2 : 4, 8>(a);
+    else if (c1 <= c2) grouped_body<TY, KIND, 2, KIND == 1 ? 1 : 2, 8>(a);
+    else grouped_body<TY, KIND, 1, KIND == 1 ? 1 : 2, 8>(a);
+}
+#define GS_GRP_AUTO(TY, KIND) \
+    extern "C" __global__ void __launch_bounds__(512) gs_k_grouped_##TY##_##KIND(GroupedArgs a) { grouped_auto<TY, KIND>(a); }
+GS_GRP_AUTO(16, 1)
+GS_GRP_AUTO(16, 2)
+GS_GRP_AUTO(18, 1)
+GS_GRP_AUTO(18, 2)
+
 #define GS_GRP_KERNEL1(TY, KIND, NT, NR, WV)                                                     \
     extern "C" __global__ void __launch_bounds__(64 * WV)                                       \
         gs_k_grouped_##TY##_##KIND##_##NT##_##NR##_##WV(GroupedArgs a) {                        \
+        grp_start<TY, 64 * WV>(a);                                                              \
         grouped_body<TY, KIND, NT, NR, WV>(a);                                                  \
     }
 #define GS_GRP_KERNEL(KIND, NT, NR, WV) GS_GRP_KERNEL1(16, KIND, NT, NR, WV) GS_GRP_KERNEL1(18, KIND, NT, NR, WV)
-// instantiated (kind, NT, NR, waves) tile shapes for IQ2_XXS (16) and IQ3_XXS (18); host.cpp
+// up to 64 pairs: (kind, NT, NR, waves) tile shapes for IQ2_XXS (16) and IQ3_XXS (18); host.cpp
 // grouped_launch keeps the same list
 GS_GRP_KERNEL(1, 1, 1, 8)
 GS_GRP_KERNEL(1, 1, 2, 8)
-GS_GRP_KERNEL(1, 2, 1, 8)
-GS_GRP_KERNEL(1, 2, 2, 8)
 GS_GRP_KERNEL(1, 1, 1, 16)
 GS_GRP_KERNEL(2, 1, 1, 8)
 GS_GRP_KERNEL(2, 1, 2, 8)
 GS_GRP_KERNEL(2, 1, 4, 8)
-GS_GRP_KERNEL(2, 2, 1, 8)
-GS_GRP_KERNEL(2, 2, 2, 8)
-GS_GRP_KERNEL(2, 2, 4, 8)
-GS_GRP_KERNEL(2, 1, 1, 16)
-GS_GRP_KERNEL(2, 1, 2, 16)
-GS_GRP_KERNEL(2, 2, 1, 16)
 
 // ---------------------------------------------------------------------------------------------
 // Activation rows -> f16 MFMA operands: out = f16(x * 2^-E), scale[row] = 2^E, with 2^E the

@@ -1220,10 +1220,10 @@ hipError_t rows_f16(const float *x, int64_t x_stride, int K, int nrows, uint16_t
 
 // kind 1 (gate/up) or 2 (down) over every tile of the layer; the grid is persistent.
 // Tile shape: NT token sub-tiles of 16 (the chunk of one expert's pairs a workgroup takes), NR row
-// sub-tiles of 16 per wave, WV waves per workgroup (one workgroup per CU shares the 65 KB decode
-// table; WV = 16 doubles the waves available to hide latency where registers allow). Larger
-// tiles stage fewer activation bytes per weight byte, but the tile count must still fill the
-// chip: take the first preferred shape whose (upper-bound) tile count is at least two per CU.
+// sub-tiles of 16 per wave, WV waves per workgroup (one workgroup per CU shares the 80 KB decode
+// tables; WV = 16 doubles the waves available to hide latency where registers allow). More than 64
+// pairs: the kernel picks its shape from the routing (grouped.hip grouped_auto). Fewer: one token
+// sub-tile, and the largest row tile whose (upper-bound) tile count is at least two per CU.
 // Instantiated shapes: grouped.hip GS_GRP_KERNEL.
 struct GrpShape {
     int nt, nr, wv;
@@ -1232,35 +1232,30 @@ hipError_t grouped_launch(int kind, int ty, GroupedArgs &a, int n_pairs, hipStre
     hipError_t e;
     DeviceCtx *c = ctx(&e);
     if (!c) return e;
-    static const std::vector<GrpShape> all1 = {{1, 1, 8}, {1, 2, 8}, {2, 1, 8}, {2, 2, 8}, {1, 1, 16}};
-    static const std::vector<GrpShape> all2 = {{1, 1, 8}, {1, 2, 8}, {1, 4, 8}, {2, 1, 8}, {2, 2, 8}, {2, 4, 8},
-                                               {1, 1, 16}, {1, 2, 16}, {2, 1, 16}};
-    // preference order (largest useful tile first), per token-chunk size
-    static const std::vector<GrpShape> pref1 = {{2, 2, 8}, {2, 1, 8}, {1, 2, 8}, {1, 1, 16}, {1, 1, 8}};
-    static const std::vector<GrpShape> pref2 = {{2, 4, 8}, {2, 2, 8}, {1, 4, 8}, {1, 2, 8}, {2, 1, 8}, {1, 1, 8}};
+    static const std::vector<GrpShape> pref1 = {{1, 2, 8}, {1, 1, 16}, {1, 1, 8}};
+    static const std::vector<GrpShape> pref2 = {{1, 4, 8}, {1, 2, 8}, {1, 1, 8}};
     const int groups = std::min(a.n_exp, n_pairs);
     auto tiles = [&](const GrpShape &sh) {
         const int64_t rbk = (int64_t)sh.wv * 16 * sh.nr;
         return (a.rows + rbk - 1) / rbk * (groups + (n_pairs + 16 * sh.nt - 1) / (16 * sh.nt));
     };
+    std::string name = "gs_k_grouped_" + std::to_string(ty) + "_" + std::to_string(kind);
     GrpShape sh{0, 0, 0};
-    for (const GrpShape &p : kind == 1 ? pref1 : pref2) {
-        if ((n_pairs <= 64) != (p.nt == 1)) continue;    // decode-sized batches: one token sub-tile
-        sh = p;
-        if (tiles(p) >= 2 * (int64_t)c->cu_count) break;
+    if (n_pairs > 64) {
+        sh = {1, kind, 8};   // its smallest tiles
+    } else {
+        for (const GrpShape &p : kind == 1 ? pref1 : pref2) {
+            sh = p;
+            if (tiles(p) >= 2 * (int64_t)c->cu_count) break;
+        }
+        name += "_" + std::to_string(sh.nt) + "_" + std::to_string(sh.nr) + "_" + std::to_string(sh.wv);
     }
-    const auto &all = kind == 1 ? all1 : all2;
-    if (std::none_of(all.begin(), all.end(),
-                     [&](const GrpShape &p) { return p.nt == sh.nt && p.nr == sh.nr && p.wv == sh.wv; }))
-        return hipErrorInvalidValue;
-    const std::string name = "gs_k_grouped_" + std::to_string(ty) + "_" + std::to_string(kind) + "_" + std::to_string(sh.nt) + "_" +
-                             std::to_string(sh.nr) + "_" + std::to_string(sh.wv);
     hipFunction_t f;
     if ((e = get_fn(c, name, &f)) != hipSuccess) return e;
     const int threads = 64 * sh.wv;
     // decode tables (80 KB, grouped.hip GS_GRP_TAB_BYTES) + four staged activation super-blocks +
     // the workgroup's bookkeeping
-    const size_t lds = 16384 + 65536 + 4 * (size_t)16 * sh.nt * 512 + GS_GRP_META_BYTES;
+    const size_t lds = 16384 + 65536 + 4 * (size_t)16 * (n_pairs > 64 ? 2 : sh.nt) * 512 + GS_GRP_META_BYTES;
     int per_cu = 1;
     {
         std::lock_guard<std::mutex> lk(g_mu);
